@@ -362,7 +362,7 @@ int read_and_clear_error(uocr_gpu_ctx* ctx) {
 
 // Engine of a forward: the one-token decode engine, the small-batch engine
 // (row tiles of <= 16 tokens, bandwidth-bound) for T <= 16, the MFMA
-// grouped GEMM for larger batches (INT8 overlays streamed as int8 rows and
+// grouped GEMMs for larger batches (INT8 overlays streamed as int8 rows and
 // dequantised in registers; under DynamicActivations the single-row groups
 // still take the small-batch engine's W8A8 path).
 enum class Engine { Decode, Batch, Mfma, Int8 };
@@ -449,14 +449,14 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
                 "small-batch engine needs widths <= 2048, expert and shared widths that are "
                 "multiples of 16 and a hidden width that is a multiple of 32");
   const bool bf16_only = (flags & UOCR_FLAG_BF16_ACTIVATIONS) != 0;
-  // Row tiles: 256 rows on the MFMA engine with BF16 weights (an expert's
-  // last tile of <= 128 rows runs as 128 x 512 items), 64 rows with INT8
-  // weights (64 x 512 items) and in the int8 mode, 16 on the small-batch
-  // engine.
-  const bool q8 = L.quant_mode != UOCR_QUANT_NONE;
-  const int bm = mfma ? (q8 ? uocr::kMfmaQ8BM : uocr::kMfmaBM)
-                      : int8 ? uocr::kI8BM : uocr::kGemvChunk;
-  const int narrow = mfma && !q8 ? uocr::kMfmaBM / 2 : 0;
+  // Row tiles: 256 rows on the MFMA engine (an expert's last tile of <= 128
+  // rows runs as 128 x 512 items), 64 rows in its weight-streaming form and
+  // in the int8 mode, 16 on the small-batch engine.
+  const bool stream = mfma && uocr::stream_preferred(L, Ti, bf16_only);
+  const int bm = stream ? uocr::kStreamBM
+                 : mfma ? uocr::kMfmaBM
+                        : int8 ? uocr::kI8BM : uocr::kGemvChunk;
+  const int narrow = mfma && !stream ? uocr::kMfmaBM / 2 : 0;
   const int tiles_bound = uocr::max_tiles(Ti, L.K, L.E, bm);
   if (tiles_bound > 65535)
     return fail(UOCR_ERR_RESOURCE, "token count too large for one forward (%zu)", T);
@@ -487,7 +487,7 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
     // engine forced at T = 1 it runs as W8A8 on the small-batch engine's
     // shared units, and the MFMA launches take the routed items only.
     const bool shared_single = mfma && T == 1 && L.quant_mode == UOCR_QUANT_DYNAMIC_ACTIVATIONS;
-    const bool overlap = mfma && ex.side && L.S > 0 && T <= kOverlapMaxTokens && !shared_single;
+    const bool overlap = mfma && !stream && ex.side && L.S > 0 && T <= kOverlapMaxTokens && !shared_single;
     if (mfma) {
       P.x_hi = S.xb;
       P.x_lo = S.xb + T * L.H;
@@ -500,9 +500,8 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
     // every value of x once anyway), so no split launch precedes it. Two
     // streams keep the split first, so that the fork comes before the
     // routing and the shared expert's GEMMs reach the CUs ahead of the
-    // routed ones (forking after the router took the 512-token INT8 layer
-    // from 0.165 to 0.199 ms; forking first with a side-stream copy of the
-    // planes measured the same as the split here).
+    // routed ones. The weight-streaming form runs both experts' items in one
+    // launch, on one stream.
     const bool fused_router = T > (size_t)uocr::kGemvChunk && uocr::router_mfma_supported(L.H);
     const bool router_planes = mfma && !planes_ready && fused_router && !overlap;
     if (mfma && !planes_ready && !router_planes) {
@@ -605,10 +604,12 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
       }
       const int lists = overlap || shared_single ? uocr::kListRouted : uocr::kListAll;
       phase_begin(ctx, kGateUp);
-      uocr::launch_mfma_gateup(L, S, P, Ti, tiles_bound, bf16_only, lists, st);
+      const auto gateup = stream ? uocr::launch_stream_gateup : uocr::launch_mfma_gateup;
+      const auto down = stream ? uocr::launch_stream_down : uocr::launch_mfma_down;
+      gateup(L, S, P, Ti, tiles_bound, bf16_only, lists, st);
       phase_end(ctx);
       phase_begin(ctx, kDown);
-      uocr::launch_mfma_down(L, S, P, Ti, tiles_bound, bf16_only, lists, st);
+      down(L, S, P, Ti, tiles_bound, bf16_only, lists, st);
       phase_end(ctx);
       if (overlap) HIP_TRY(hipStreamWaitEvent(st, ex.join, 0), "join wait");
     } else {

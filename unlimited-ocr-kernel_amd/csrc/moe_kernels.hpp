@@ -189,8 +189,8 @@ void launch_int8_dynamic(const int8_t* q, const float* sc, int rows, int cols, c
                          hipStream_t s);
 void gemv_init_attributes();
 
-// gemm.hip: MFMA grouped GEMM engine. Activations enter as bf16 planes
-// (hi, and lo for FP32-class precision).
+// gemm.hip: MFMA grouped GEMM engine (BF16 weights, larger batches).
+// Activations enter as bf16 planes (hi, and lo for FP32-class precision).
 struct MfmaPlanes {
   uint16_t* x_hi;   // [H/32][T][32] (k-blocked)
   uint16_t* x_lo;
@@ -208,7 +208,6 @@ void launch_mfma_gateup(const DeviceLayer& L, const Scratch& S, const MfmaPlanes
 void launch_mfma_down(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
                       int tiles_bound, bool bf16_only, int lists, hipStream_t s);
 constexpr int kMfmaBM = 256;
-constexpr int kMfmaQ8BM = 64;  // INT8 weights: 64-row tiles, 64 x 512 items
 void mfma_init_attributes();
 // out = `groups` row-major [N, K] matrices (elem_bytes 1 or 2, K % 32 == 0,
 // matrix g at g * N * K) as k-blocked panels [K/32][N][32].
@@ -218,6 +217,16 @@ void launch_transpose_f32(const float* in, float* out, int rows, int cols, int g
                           hipStream_t s);
 void launch_panelize(const void* in, void* out, int elem_bytes, int N, int K, int groups,
                      hipStream_t s);
+
+// stream.hip: the weight-streaming form of the same GEMMs (the same planes in
+// and out; row tiles of kStreamBM), for every INT8 batch and for BF16 batches
+// of small groups.
+constexpr int kStreamBM = 64;
+bool stream_preferred(const DeviceLayer& L, int T, bool bf16_only);
+void launch_stream_gateup(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
+                          int tiles_bound, bool bf16_only, int lists, hipStream_t s);
+void launch_stream_down(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
+                        int tiles_bound, bool bf16_only, int lists, hipStream_t s);
 
 // gemm_i8.hip: int8 x int8 grouped GEMM with int32 block accumulation (the
 // opt-in UOCR_FLAG_INT8_MFMA mode). Activations enter quantised per 32-block.
