@@ -586,7 +586,8 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
       uocr::launch_i8_down(L, S, P, Ti, tiles_bound, st);
       phase_end(ctx);
     } else if (mfma) {
-      if (L.quant_mode == UOCR_QUANT_DYNAMIC_ACTIVATIONS) {
+      const bool stream_singles = stream && uocr::stream_takes_singles(L);
+      if (L.quant_mode == UOCR_QUANT_DYNAMIC_ACTIVATIONS && (!stream_singles || shared_single)) {
         // W8A8 for groups of one row (src/decoder/mod.rs:103-104): the
         // small-batch engine's single-row pass on this stream (hidden rows
         // in S.gu; the W8A8 trace's hidden rows written by the pass itself).
@@ -594,18 +595,22 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
         // lengthened the stream that ends the layer (512-token W8A8 layer
         // 0.162 -> 0.171 ms).
         phase_begin(ctx, kGateUp);
-        uocr::launch_singles_gateup(L, S, Ti, st);
+        if (!stream_singles) uocr::launch_singles_gateup(L, S, Ti, st);
         if (shared_single) uocr::launch_batch_gateup(L, S, Ti, tiles_bound, bm, st, true);
         phase_end(ctx);
         phase_begin(ctx, kDown);
-        uocr::launch_singles_down(L, S, Ti, st);
+        if (!stream_singles) uocr::launch_singles_down(L, S, Ti, st);
         if (shared_single) uocr::launch_batch_down(L, S, Ti, tiles_bound, bm, st, true);
         phase_end(ctx);
       }
       const int lists = overlap || shared_single ? uocr::kListRouted : uocr::kListAll;
       phase_begin(ctx, kGateUp);
-      const auto gateup = stream ? uocr::launch_stream_gateup : uocr::launch_mfma_gateup;
-      const auto down = stream ? uocr::launch_stream_down : uocr::launch_mfma_down;
+      const auto gateup = stream_singles ? uocr::launch_stream_singles_gateup
+                          : stream       ? uocr::launch_stream_gateup
+                                         : uocr::launch_mfma_gateup;
+      const auto down = stream_singles ? uocr::launch_stream_singles_down
+                        : stream       ? uocr::launch_stream_down
+                                       : uocr::launch_mfma_down;
       gateup(L, S, P, Ti, tiles_bound, bf16_only, lists, st);
       phase_end(ctx);
       phase_begin(ctx, kDown);

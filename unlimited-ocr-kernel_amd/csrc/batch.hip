@@ -26,6 +26,7 @@
 #include "moe_kernels.hpp"
 #include "routing.hpp"
 #include "rowdot.hpp"
+#include "stream.hpp"
 
 namespace uocr {
 
@@ -58,6 +59,10 @@ __host__ __device__ inline int seg_of(int W) {
   return W <= kSegK ? W : ((W + 1) / 2 + kQBlock - 1) / kQBlock * kQBlock;
 }
 __host__ __device__ inline int down_units(int H, int W) { return W <= kSegK ? H / 32 : H / 16; }
+
+// A thread's number within its unit's 256: a workgroup's own, or one of the
+// two units that a 512-thread workgroup runs side by side.
+__device__ __forceinline__ int unit_tid() { return threadIdx.x & 255; }
 
 struct Unit {
   int g, r0, n, group_rows, slice;
@@ -171,7 +176,8 @@ struct BatchSmem {
 template <typename RowOf>
 __device__ __forceinline__ void stage_tile(BatchSmem& sm, int b0, int nb, int K, int ld,
                                            RowOf row_of) {
-  if (threadIdx.x < nb) sm.rows[threadIdx.x] = row_of(b0 + threadIdx.x);
+  const int tid = unit_tid();
+  if (tid < nb) sm.rows[tid] = row_of(b0 + tid);
   __syncthreads();
   const int vec = ld / 4, kvec = K / 4;
   const int total = nb * vec;
@@ -180,14 +186,14 @@ __device__ __forceinline__ void stage_tile(BatchSmem& sm, int b0, int nb, int K,
     u32x4 v[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      const int at = base + threadIdx.x + i * 256;
+      const int at = base + tid + i * 256;
       const int t = at / vec, c = at - t * vec;
       v[i] = u32x4{0u, 0u, 0u, 0u};
       if (at < total && c < kvec) v[i] = reinterpret_cast<const u32x4*>(sm.rows[t])[c];
     }
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      const int at = base + threadIdx.x + i * 256;
+      const int at = base + tid + i * 256;
       if (at < total) reinterpret_cast<u32x4*>(sm.x)[at] = v[i];
     }
   }
@@ -232,7 +238,7 @@ __device__ __forceinline__ void tile_dot(const DeviceLayer& L, const Scratch& S,
       stage_tile(sm, 0, 1, cols, ld, row_of);
       // The zero columns quantise to zero blocks, so every block a segment
       // can reach is defined.
-      quantize_lds_waves(sm.x, ld, sm.xq, sm.xs, threadIdx.x >> 6, blockDim.x >> 6, lane, S.err);
+      quantize_lds_waves(sm.x, ld, sm.xq, sm.xs, unit_tid() >> 6, 4, lane, S.err);
       __syncthreads();
       float r0, r1;
       dot_rows_as<kW8A8>(P, K, sm.x, sm.xq, sm.xs, r0, r1, xb_off, sums);
@@ -280,7 +286,7 @@ template <int KIND, int KH, bool DYN, bool SINGLE = false>
 __device__ __forceinline__ void gateup_body(const DeviceLayer& L, const Scratch& S, BatchSmem& sm,
                                             const Unit& u) {
   const int W = L.width(u.g);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = unit_tid() >> 6, lane = threadIdx.x & 63;
   const int k = 16 * u.slice + 4 * wave + (lane >> 4);
   const int ra = gate_row(k);
   RowPair<KIND, KH> P;
@@ -354,7 +360,7 @@ template <int KIND, bool HALVES, bool DYN, bool SINGLE = false>
 __device__ __forceinline__ void down_body(const DeviceLayer& L, const Scratch& S, BatchSmem& sm,
                                           const Unit& u) {
   const int W = L.width(u.g);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = unit_tid() >> 6, lane = threadIdx.x & 63;
   const int seg = seg_of(W);
   const int ra = HALVES ? 16 * u.slice + 4 * wave + (lane >> 4) : 32 * u.slice + 8 * wave + (lane >> 4);
   const int rb = HALVES ? ra : ra + 4;
@@ -434,7 +440,6 @@ __attribute__((amdgpu_waves_per_eu(3))) void batch_down_kernel(
 // routing), and the shared down units at the head of the gate/up launch;
 // the down launch then holds routed units only. Otherwise (INT8 layers
 // only) the shared units head the gate/up and down launches.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kMfmaSharedRows = 16;
@@ -726,6 +731,54 @@ __attribute__((amdgpu_waves_per_eu(3))) void singles_down_kernel(DeviceLayer L, 
   }
 }
 
+// The streaming GEMM of a DynamicActivations layer with the single-row pass of
+// the same projection in the workgroups from n_stream on (512 threads: two
+// units side by side, in step, since every single-row unit passes the same
+// barriers; an odd last unit runs twice, with the same results). A launch of
+// its own cost each pass 4 us even where no group has one row, and up to 20
+// where many have: one W8A8 layer, even / Zipf / hot routing, 17 tokens 89 ->
+// 71 / 68 -> 56 / 67 -> 53 us, 61 tokens 73 -> 69 / 86 -> 73 / 96 -> 77, 273
+// tokens 96 -> 95 / 106 -> 102 / 112 -> 112. 512 workgroups: with 128 of them
+// 17 tokens took 96 / 64 / 63 us, with 256 78 / 58 / 55.
+constexpr int kStreamSingles = 512;  // workgroups
+
+template <int KR, int KSH, bool SPLIT, bool GATEUP>
+__global__ __launch_bounds__(kStreamThreads, 4) void stream_singles_kernel(DeviceLayer L, Scratch S,
+                                                                           MfmaPlanes P, int T,
+                                                                           int lists, int n_stream) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int id = (int)blockIdx.x;
+  if (id < n_stream) {
+    stream_work<KR, KSH, SPLIT, GATEUP, true>(L, S, P, T, lists, id, lds);
+    return;
+  }
+  const int half = threadIdx.x >> 8;
+  BatchSmem& sm = reinterpret_cast<BatchSmem*>(lds)[half];
+  const unsigned long long m = single_groups(L, S);
+  const int ur = GATEUP ? (L.I + 15) / 16 : L.H / 32, n = __popcll(m) * ur;
+  for (int b = id - n_stream; 2 * b < n; b += kStreamSingles) {
+    const Unit u = single_unit(m, ur, min(2 * b + half, n - 1));
+    if constexpr (GATEUP)
+      gateup_body<kInt8, 1280, true, true>(L, S, sm, u);
+    else
+      down_body<kInt8, false, true, true>(L, S, sm, u);
+    __syncthreads();  // this unit's LDS consumed before the next is staged
+  }
+}
+
+template <bool GATEUP>
+void launch_stream_with_singles(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
+                                int tiles_bound, bool bf16_only, int lists, hipStream_t s) {
+  stream_select<GATEUP>(
+      L, T, tiles_bound, bf16_only, lists,
+      [&](auto kr, auto ksh, auto split, auto q8, unsigned blocks, size_t lds) {
+        if constexpr (q8())
+          stream_singles_kernel<kr(), ksh(), split(), GATEUP>
+              <<<dim3(blocks + kStreamSingles), dim3(kStreamThreads),
+                 std::max(lds, 2 * sizeof(BatchSmem)), s>>>(L, S, P, T, lists, (int)blocks);
+      });
+}
+
 // ------------------------------------------------------------- small router
 
 // Routing of T <= 16 tokens in one launch. Workgroup (b, p) dots router
@@ -979,6 +1032,23 @@ void launch_singles_down(const DeviceLayer& L, const Scratch& S, int T, hipStrea
     singles_down_kernel<false><<<grid, block, 0, s>>>(L, S);
   else
     singles_down_kernel<true><<<grid, block, 0, s>>>(L, S);
+}
+
+// The single-row units that fit the streaming kernel's registers: hidden rows
+// of at most 1280 values, whole down rows.
+bool stream_takes_singles(const DeviceLayer& L) {
+  return L.quant_mode == kQuantDynamic && L.H <= 1280 && L.I <= kSegK;
+}
+
+void launch_stream_singles_gateup(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P,
+                                  int T, int tiles_bound, bool bf16_only, int lists,
+                                  hipStream_t s) {
+  launch_stream_with_singles<true>(L, S, P, T, tiles_bound, bf16_only, lists, s);
+}
+
+void launch_stream_singles_down(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
+                                int tiles_bound, bool bf16_only, int lists, hipStream_t s) {
+  launch_stream_with_singles<false>(L, S, P, T, tiles_bound, bf16_only, lists, s);
 }
 
 void launch_batch_down(const DeviceLayer& L, const Scratch& S, int T, int tiles_bound, int mchunk,

@@ -228,6 +228,14 @@ void launch_stream_gateup(const DeviceLayer& L, const Scratch& S, const MfmaPlan
 void launch_stream_down(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
                         int tiles_bound, bool bf16_only, int lists, hipStream_t s);
 
+// The same launches with the single-row W8A8 groups of a DynamicActivations
+// layer (launch_singles_gateup / _down) in workgroups of their own (batch.hip).
+bool stream_takes_singles(const DeviceLayer& L);
+void launch_stream_singles_gateup(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P,
+                                  int T, int tiles_bound, bool bf16_only, int lists, hipStream_t s);
+void launch_stream_singles_down(const DeviceLayer& L, const Scratch& S, const MfmaPlanes& P, int T,
+                                int tiles_bound, bool bf16_only, int lists, hipStream_t s);
+
 // gemm_i8.hip: int8 x int8 grouped GEMM with int32 block accumulation (the
 // opt-in UOCR_FLAG_INT8_MFMA mode). Activations enter quantised per 32-block.
 struct I8Planes {
