@@ -480,8 +480,6 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
     // kOverlapMaxTokens tokens.
     constexpr size_t kOverlapMaxTokens = 2048;
     uocr::MfmaPlanes P{};
-    // (Under DynamicActivations the small-batch engine's single-row pass on
-    // this stream touches only routed rows' hidden and output buffers.)
     // Under DynamicActivations one token makes the shared expert a
     // single-row group as well (src/decoder/mod.rs:103-104): with the MFMA
     // engine forced at T = 1 it runs as W8A8 on the small-batch engine's
@@ -588,12 +586,10 @@ int enqueue_experts(const Exec& ex, const uocr_moe_layer* layer, const float* x,
     } else if (mfma) {
       const bool stream_singles = stream && uocr::stream_takes_singles(L);
       if (L.quant_mode == UOCR_QUANT_DYNAMIC_ACTIVATIONS && (!stream_singles || shared_single)) {
-        // W8A8 for groups of one row (src/decoder/mod.rs:103-104): the
-        // small-batch engine's single-row pass on this stream (hidden rows
-        // in S.gu; the W8A8 trace's hidden rows written by the pass itself).
-        // On the second stream, after the shared expert's GEMMs, it
-        // lengthened the stream that ends the layer (512-token W8A8 layer
-        // 0.162 -> 0.171 ms).
+        // W8A8 for groups of one row (src/decoder/mod.rs:103-104), where the
+        // streaming launches below do not take them: the small-batch engine's
+        // single-row pass (hidden rows in S.gu; the W8A8 trace's hidden rows
+        // written by the pass itself).
         phase_begin(ctx, kGateUp);
         if (!stream_singles) uocr::launch_singles_gateup(L, S, Ti, st);
         if (shared_single) uocr::launch_batch_gateup(L, S, Ti, tiles_bound, bm, st, true);
