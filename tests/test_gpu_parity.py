@@ -753,8 +753,8 @@ def test_int8_mfma(ctx, full_int8, full_dynamic, T):
     """INT8 overlays on the MFMA engine: int8 rows (exact in bf16) and block
     scales are streamed; each 32-deep block's partial product with the
     activation planes (hi + lo for the FP32 class, hi for BF16 activations)
-    is scaled by its block scale into the f32 accumulator. 64-row tiles run
-    as 64 x 512 items (T = 512 puts ~48 rows in each expert). Under
+    is scaled by its block scale into the f32 accumulator. Items are up to 64
+    rows x 256 columns (T = 512 puts ~48 rows in each expert). Under
     DynamicActivations the groups of one row take the W8A8 path
     (src/decoder/mod.rs:103-104); T = 17 and 64 leave several such groups
     among 64 experts."""
@@ -775,26 +775,29 @@ def test_int8_mfma(ctx, full_int8, full_dynamic, T):
 
 @pytest.mark.parametrize("kind", ["bf16", "int8", "w8a8"])
 def test_one_stream_matches_two_streams(ctx, full_bf16, full_int8, full_dynamic, kind):
-    """Up to 2048 tokens the shared expert's GEMMs run on a second stream
-    after a split of the input into bf16 planes; on one stream (phase
-    timing on) the router writes those planes itself. Under
-    DynamicActivations the single-row pass runs on the main stream after
-    the dispatch, before the routed GEMMs, with its hidden rows in its own
-    scratch rows by dispatched position (24 tokens leave 15 groups of one
-    row). Same bits either way, in both activation classes."""
-    case = {"bf16": full_bf16, "int8": full_int8, "w8a8": full_dynamic}[kind]
-    T = 24 if kind == "w8a8" else 512
+    """BF16 batches on the 256 x 256 tiles (here 1531 tokens: more than 896, or
+    640 with BF16 activations, and not a multiple of 256) run the shared
+    expert's GEMMs on a second stream up to 2048 tokens, after a split of the
+    input into bf16 planes; on one stream (phase timing on) the router writes
+    those planes itself. INT8 layers run both experts in one launch on one
+    stream, under DynamicActivations with the single-row units in workgroups of
+    their own (24 tokens leave 15 groups of one row): events between the
+    launches change nothing. Same bits either way, in both activation classes."""
+    case, T = {"bf16": (full_bf16, 1531), "int8": (full_int8, 512),
+               "w8a8": (full_dynamic, 24)}[kind]
     x = syn.activations(T, 1280, seed=811)
     for flags, name in ((0, "fp32-class"), (um.FLAG_BF16_ACTIVATIONS, "bf16 activations")):
-        say(f"{kind} T={T} {name}: two streams vs one")
+        say(f"{kind} T={T} {name}: phase timing off vs on")
         y2, tr = case.run(ctx, x, flags=um.FLAG_FORCE_MFMA | flags)
         if kind == "w8a8":
             assert (np.diff(tr["expert_offsets"]) == 1).sum() == 15
         ctx.set_timing("all")
         try:
             y1, _ = case.run(ctx, x, flags=um.FLAG_FORCE_MFMA | flags)
+            split = ctx.timings()["split"][0]
         finally:
             ctx.set_timing(())
+        assert split == 0, "one stream: the router writes the planes"
         assert np.array_equal(y1.view(np.uint32), y2.view(np.uint32)), name
 
 

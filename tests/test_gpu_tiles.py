@@ -1,18 +1,54 @@
-"""Which grouped GEMM a BF16 batch takes: the weight-streaming kernel or the
-256 x 256 tiles."""
+"""The 256 x 256 grouped GEMM at the edges of its tiles, and which BF16 batches
+take it: those above 896 tokens (640 with BF16 activations), and above a number
+of operations in wide layers; the rest take the weight-streaming kernel."""
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
 import uocr_moe as um  # noqa: E402
-from test_gpu_parity import ctx  # noqa: E402,F401
+from test_gpu_parity import Case, check_layer, ctx  # noqa: E402,F401
+from test_gpu_stream import BF16_CLASS, FP32_CLASS  # noqa: E402
 from uocr_moe import synthetic as syn  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
+BF16 = um.FLAG_BF16_ACTIVATIONS
+# Two experts that every token takes (each group has T rows), and eight of which
+# it takes two (uneven groups). Column tiles of 256 and 512 that are not full, 2,
+# 6 and 10 stages of K.
+SHAPES = [dict(hidden=64, inter=64, experts=2, shared=2),
+          dict(hidden=320, inter=192, experts=8, shared=1)]
+
+
+@pytest.mark.parametrize("T,flags", [(897, 0), (1025, 0), (1531, 0), (641, BF16), (1025, BF16),
+                                     (1531, BF16), (2305, BF16)])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_tile_edges(ctx, shape, T, flags):  # noqa: F811
+    """Last row tiles of 1, 129 and 251 rows (each form has its own items for
+    128 or fewer), up to 2048 tokens with the shared expert on a second stream;
+    BF16 activations have square items only beyond that."""
+    case = Case(ctx, SHAPES[shape], 2, seed=950 + shape)
+    x = syn.activations(T, SHAPES[shape]["hidden"], seed=960 + T)
+    print(f"tiles shape={shape} T={T} flags={flags}", flush=True)
+    y = check_layer(case, ctx, x, tol=BF16_CLASS if flags else FP32_CLASS, flags=flags)
+    # A row does not depend on its place or on the other rows of its tile.
+    back, _ = case.run(ctx, np.ascontiguousarray(x[::-1]), flags)
+    assert np.array_equal(back[::-1], y)
+
+
+@pytest.mark.parametrize("T,flags", [(896, 0), (897, 0), (640, BF16), (641, BF16)])
+def test_last_streaming_and_first_tiled_batch(ctx, T, flags):  # noqa: F811
+    """Row tiles, work lists and streams change from one size to the next."""
+    shape = dict(hidden=192, inter=128, experts=16, shared=3)
+    case = Case(ctx, shape, 4, seed=970)
+    print(f"engine boundary T={T} flags={flags}", flush=True)
+    check_layer(case, ctx, syn.activations(T, 192, seed=971),
+                tol=BF16_CLASS if flags else FP32_CLASS, flags=flags)
+
 
 @pytest.mark.parametrize("T,larger,flags", [(832, 1024, 0),
-                                            (608, 672, um.FLAG_BF16_ACTIVATIONS)],
+                                            (608, 672, BF16)],
                          ids=["fp32-class", "bf16-activations"])
 def test_wide_layer_takes_the_tiles(ctx, T, larger, flags):  # noqa: F811
     """A wide layer (23 M multiply-adds a token; the streaming kernel was up to
