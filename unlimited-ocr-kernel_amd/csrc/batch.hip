@@ -454,21 +454,6 @@ union SharedSmem {
   MfmaUnitSmem m;
 };
 
-// Eight int8 weights as bf16 (the f32 of a small integer has a zero low
-// half, so its bf16 is the high half).
-__device__ __forceinline__ bf16x8 widen_q8(u32x2 q) {
-  uint32_t hp[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint32_t word = j < 2 ? q.x : q.y;
-    const int s0 = 16 * (j & 1);
-    const float w0 = (float)(int8_t)((word >> s0) & 0xffu);
-    const float w1 = (float)(int8_t)((word >> (s0 + 8)) & 0xffu);
-    hp[j] = __builtin_amdgcn_perm(__float_as_uint(w1), __float_as_uint(w0), 0x07060302u);
-  }
-  return __builtin_bit_cast(bf16x8, u32x4{hp[0], hp[1], hp[2], hp[3]});
-}
-
 // Rows ra (and, with NSET = 2, rb) -- this lane's column of each row set --
 // of a k-blocked panel [K/32][rows][32] (BF16, or INT8 with row-major block
 // scales [rows][K/32]), dotted with activation row xrow: with F32X, FP32
@@ -548,13 +533,13 @@ __device__ __forceinline__ void mfma_rows_dot(const void* panel, const float* sc
     }
     if constexpr (kQ8) {
       const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-      const bf16x8 wa = widen_q8(qa[i]);
+      const bf16x8 wa = widen_int8x8(qa[i].x, qa[i].y);
       f32x4 pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, wa, z, 0, 0, 0);
       pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, wa, pa, 0, 0, 0);
 #pragma unroll
       for (int r = 0; r < 4; r++) acc_a[r] = __builtin_fmaf(pa[r], sa[i], acc_a[r]);
       if constexpr (NSET == 2) {
-        const bf16x8 wb = widen_q8(qb[i]);
+        const bf16x8 wb = widen_int8x8(qb[i].x, qb[i].y);
         f32x4 pb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, wb, z, 0, 0, 0);
         pb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, wb, pb, 0, 0, 0);
 #pragma unroll
@@ -734,8 +719,8 @@ __attribute__((amdgpu_waves_per_eu(3))) void singles_down_kernel(DeviceLayer L, 
 // The streaming GEMM of a DynamicActivations layer with the single-row pass of
 // the same projection in the workgroups from n_stream on (512 threads: two
 // units side by side, in step, since every single-row unit passes the same
-// barriers; an odd last unit runs twice, with the same results). A launch of
-// its own cost each pass 4 us even where no group has one row, and up to 20
+// barriers; a group's units are even in number, H and I being multiples of 64).
+// A launch of its own cost each pass 4 us even where no group has one row, and up to 20
 // where many have: one W8A8 layer, even / Zipf / hot routing, 17 tokens 89 ->
 // 71 / 68 -> 56 / 67 -> 53 us, 61 tokens 73 -> 69 / 86 -> 73 / 96 -> 77, 273
 // tokens 96 -> 95 / 106 -> 102 / 112 -> 112. 512 workgroups: with 128 of them
@@ -757,7 +742,7 @@ __global__ __launch_bounds__(kStreamThreads, 4) void stream_singles_kernel(Devic
   const unsigned long long m = single_groups(L, S);
   const int ur = GATEUP ? (L.I + 15) / 16 : L.H / 32, n = __popcll(m) * ur;
   for (int b = id - n_stream; 2 * b < n; b += kStreamSingles) {
-    const Unit u = single_unit(m, ur, min(2 * b + half, n - 1));
+    const Unit u = single_unit(m, ur, 2 * b + half);
     if constexpr (GATEUP)
       gateup_body<kInt8, 1280, true, true>(L, S, sm, u);
     else

@@ -72,14 +72,6 @@ __device__ __forceinline__ void buffer_load_lds16(i32x4 rsrc, uint32_t lds_addr,
                : "memory");
 }
 
-// The same for 4 bytes per lane (lane l's dword lands at M0 + 4 l).
-__device__ __forceinline__ void buffer_load_lds4(i32x4 rsrc, uint32_t lds_addr, uint32_t voffset) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               :
-               : "s"(lds_addr), "v"(voffset), "s"(rsrc)
-               : "memory");
-}
-
 __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t bytes) {
   const unsigned long long a = reinterpret_cast<unsigned long long>(base);
   i32x4 r;

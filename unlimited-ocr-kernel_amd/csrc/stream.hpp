@@ -408,7 +408,8 @@ void stream_shape(const DeviceLayer& L, int T, int tiles_bound, bool bf16_only, 
     if ((GATEUP ? L.H : L.I) / 64 % KR)
       return stream_shape<1, KSH, GATEUP>(L, T, tiles_bound, bf16_only, lists, go);
   }
-  if constexpr (KSH > 1) {
+  // (Where I / 64 is even, so is S / 64: S is a multiple of I.)
+  if constexpr (KSH > 1 && KR == 1) {
     if ((GATEUP ? L.H : L.S) / 64 % KSH)
       return stream_shape<KR, 1, GATEUP>(L, T, tiles_bound, bf16_only, lists, go);
   }
