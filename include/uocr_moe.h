@@ -257,7 +257,11 @@ void uocr_moe_layer_destroy(uocr_moe_layer* layer);
  * sum over each row's top-k experts, ascending id, of p * expert(x).
  * x and y are device pointers (FP32 row-major [T,H]). Enqueued on the
  * context stream; the call returns once the work is queued. Device-side
- * errors surface at uocr_gpu_ctx_synchronize. T == 0 is a no-op. */
+ * errors surface at uocr_gpu_ctx_synchronize. T == 0 is a no-op.
+ * Equal calls give equal bits. A row's last bits depend on T as well, which
+ * chooses the engine and how its sums are split (see the tolerance classes
+ * above): the same row in a batch of 1, 16, 32, 33, 256, 257 or 897 tokens is
+ * summed in different orders. */
 int uocr_moe_forward_async(uocr_gpu_ctx* ctx, const uocr_moe_layer* layer, const float* x,
                            size_t T, float* y, uint32_t flags, const uocr_moe_trace* trace);
 /* The same, then synchronize: errors are reported by this call. */

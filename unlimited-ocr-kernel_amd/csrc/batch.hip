@@ -1019,8 +1019,12 @@ void launch_singles_down(const DeviceLayer& L, const Scratch& S, int T, hipStrea
     singles_down_kernel<true><<<grid, block, 0, s>>>(L, S);
 }
 
-// The single-row units that fit the streaming kernel's registers: hidden rows
-// of at most 1280 values, whole down rows.
+// The widths whose single-row units the streaming launches take: hidden rows of
+// at most 1280 values, whole down rows. The down units fit the launch's 128
+// VGPRs; the gate/up unit takes 132 in a kernel of its own, and here its
+// workgroups spill: one VGPR, stored once ahead of their units and read back
+// where block sums are traced, and 12 SGPRs to lanes of another (8 bytes of
+// scratch a lane). The streaming items have branched off before.
 bool stream_takes_singles(const DeviceLayer& L) {
   return L.quant_mode == kQuantDynamic && L.H <= 1280 && L.I <= kSegK;
 }

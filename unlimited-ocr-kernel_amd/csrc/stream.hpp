@@ -21,14 +21,17 @@
 // 55 us (5.5 TB/s, against 88 us of 128 x 512 items, with the shared expert's
 // 122 us on a second stream); down, 151 MB in 35 us: one CU takes in 25-30
 // B/ns, and the workgroups do not divide evenly over 256 CUs. 512 tokens INT8
-// gate/up 62 us (94): without its weight loads it still takes 65, without its
-// activation loads 69 (of 74 then), the widening (24 VALU instructions per 32
-// rows and 32-block) and scaling (8 per 16 tokens) beside the MFMAs. Measured
-// and not kept: 32 x 32 MFMA tiles (up to 25% more padding: 512 tokens 122
-// against 116 us a layer); 4 waves of 64 features (151 us); 7, 10 or 14 waves a
-// workgroup, so that items divide the CUs evenly (one 14-wave workgroup a CU:
-// gate/up 53 against 58 us at 61 tokens, but 80 against 72 us at 512, its
-// waves in step).
+// gate/up, 170 MB in 62-65 us (94): the matrix cores are busy 0.28 of the time
+// and the VALU 0.41 (24 instructions of widening per 32 rows and 32-block, 8 of
+// scaling per 16 tokens), so neither they nor HBM set the time; the waves wait.
+// (An earlier form that took 74 us took 65 without its weight loads and 69
+// without its activation loads.) What they wait for was not taken apart: a
+// fragment is read from LDS right before the product that needs it, and each
+// item starts with four dependent reads for its 20 (14) chunks. Measured and not
+// kept: 32 x 32 MFMA tiles (up to 25% more padding: 512 tokens 122 against 116
+// us a layer); 4 waves of 64 features (151 us); 7, 10 or 14 waves a workgroup,
+// so that items divide the CUs evenly (one 14-wave workgroup a CU: gate/up 53
+// against 58 us at 61 tokens, but 80 against 72 us at 512, its waves in step).
 #pragma once
 
 #include <algorithm>
