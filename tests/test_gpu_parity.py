@@ -314,6 +314,32 @@ def test_widths_beyond_small_batch(ctx, T, quant):
     assert e.value.status == um.UNSUPPORTED
 
 
+# Hidden widths beyond 2048: the combine takes a row in column slices of 2048
+# (here two and three, the last of 64 columns), every batch the grouped GEMMs
+# and the unfused router.
+@pytest.mark.parametrize("hidden", [2112, 4160])
+@pytest.mark.parametrize("quant", [orc.QUANT_NONE, orc.QUANT_WEIGHTS_ONLY])
+def test_hidden_beyond_2048(ctx, hidden, quant):
+    shape = dict(hidden=hidden, inter=64, experts=4, shared=1)
+    case = Case(ctx, shape, 2, seed=100 + quant, quant=quant)
+    for T in (1, 5, 17, 130, 897):
+        say(f"hidden {hidden} T={T} quant={quant}")
+        x = syn.activations(T, hidden, seed=110 + T)
+        check_layer(case, ctx, x)
+        check_layer(case, ctx, x, tol=BF16_TOL, flags=um.FLAG_BF16_ACTIVATIONS)
+    # The block form: x + experts(rms_norm(x)), the residual in the same slices.
+    say(f"hidden {hidden} block T={T} quant={quant}")
+    normed = orc.rms_norm(x, orc.bf16_to_f32(case.w["norm_weight"]), 1e-6)
+    out, rtr = orc.moe_experts(case.orc, normed, trace=True)
+    srt = np.sort(rtr.logits, axis=1)[:, ::-1]
+    keep = srt[:, 1] - srt[:, 2] >= 1e-5
+    xd = dev(x)
+    yd = torch.full_like(xd, float("nan"))
+    um.block_forward(ctx, [case.layer], xd, yd)
+    got = yd.cpu().numpy()
+    assert np.all(np.isfinite(got)) and normwise(got[keep], (x + out)[keep]) <= FP32_TOL
+
+
 @pytest.fixture(scope="module")
 def full_bf16(ctx):
     return Case(ctx, FULL, 6, seed=0)

@@ -24,14 +24,16 @@ __device__ __forceinline__ float4 load4(const float* __restrict__ row, int i) {
   }
 }
 
-// Combine, then (NORM) the next layer's RMSNorm of the result. Y16: the
-// expert outputs (routed and shared) are bf16 rows (BF16 activations).
+// Combine, then (NORM, rows up to kRowWidth wide) the next layer's RMSNorm of
+// the result. Y16: the expert outputs (routed and shared) are bf16 rows (BF16
+// activations). Workgroup (t, s) takes columns kRowWidth s .. of row t.
 template <bool NORM, bool Y16>
 __global__ __launch_bounds__(kRowThreads) void combine_kernel(
     const float* __restrict__ ys, const float* __restrict__ y, const int* __restrict__ ids,
     const float* __restrict__ w, const int* __restrict__ inv_pos, const float* __restrict__ residual,
     int H, int K, float* __restrict__ out, RowNorm nn, int* err) {
   const int t = blockIdx.x;
+  const int c0 = NORM ? 0 : (int)blockIdx.y * kRowWidth;
   int e[8], pos[8];
   float p[8];
 #pragma unroll
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(kRowThreads) void combine_kernel(
   float4 sv[kRowChunks], rv[kRowChunks], v[kRowChunks][8];
 #pragma unroll
   for (int it = 0; it < kRowChunks; it++) {
-    const int i = (threadIdx.x + kRowThreads * it) * 4;
+    const int i = c0 + (threadIdx.x + kRowThreads * it) * 4;
     if (i >= H) break;
     sv[it] = load4<Y16>(ys + t * rs, i);
 #pragma unroll
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(kRowThreads) void combine_kernel(
   float4 row[kRowChunks];
 #pragma unroll
   for (int it = 0; it < kRowChunks; it++) {
-    const int i = (threadIdx.x + kRowThreads * it) * 4;
+    const int i = c0 + (threadIdx.x + kRowThreads * it) * 4;
     if (i >= H) break;
     float4 acc = sv[it];
 #pragma unroll
@@ -200,9 +202,10 @@ void launch_combine(const Scratch& S, const float* residual, int T, int H, int K
 #undef UOCR_COMBINE_WAVE
     return;
   }
+  const dim3 grid(T, next ? 1 : (H + kRowWidth - 1) / kRowWidth);
 #define UOCR_COMBINE(NORM, Y16)                                                               \
-  combine_kernel<NORM, Y16><<<T, kRowThreads, 0, s>>>(S.ys, S.y, S.topk_ids, S.topk_w,         \
-                                                      S.inv_pos, residual, H, K, out, nn, S.err)
+  combine_kernel<NORM, Y16><<<grid, kRowThreads, 0, s>>>(S.ys, S.y, S.topk_ids, S.topk_w,      \
+                                                         S.inv_pos, residual, H, K, out, nn, S.err)
   if (next && y16)
     UOCR_COMBINE(true, true);
   else if (next)
@@ -276,7 +279,7 @@ __global__ __launch_bounds__(256) void rms_norm_wide_kernel(const float* __restr
   for (int i = threadIdx.x; i < width; i += blockDim.x) out[(size_t)row * width + i] = in[i] * scale * w[i];
 }
 
-bool row_norm_fusable(int width) { return width % 4 == 0 && width <= kRowThreads * kRowChunks * 4; }
+bool row_norm_fusable(int width) { return width % 4 == 0 && width <= kRowWidth; }
 bool row_norm_wave(int width) { return width % 4 == 0 && width <= kWaveRowWidth; }
 
 void launch_rms_norm(const float* x, int rows, int width, const RowNorm& nn, int* err,

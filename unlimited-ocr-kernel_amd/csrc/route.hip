@@ -21,7 +21,7 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const float* __restric
   const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (e >= E) return;
   const uint32_t* row = reinterpret_cast<const uint32_t*>(w + (size_t)e * H);
-  const int pairs = H / 2;  // H is a multiple of 128
+  const int pairs = H / 2;  // H is a multiple of 64
   float acc[TMAX];
 #pragma unroll
   for (int t = 0; t < TMAX; t++) acc[t] = 0.0f;

@@ -11,7 +11,7 @@ namespace uocr {
 
 // One row (token) per workgroup of 256 threads; thread i holds float4
 // chunks i and i + 256 of the row (widths up to 2048).
-constexpr int kRowThreads = 256, kRowChunks = 2;
+constexpr int kRowThreads = 256, kRowChunks = 2, kRowWidth = 4 * kRowThreads * kRowChunks;
 
 // RMSNorm of a row held as float4 chunks (src/cpu/ops.rs:362-423, center =
 // false): variance = sum(v^2) / W, scale = 1 / sqrt(variance + eps),
