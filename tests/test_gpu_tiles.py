@@ -47,17 +47,18 @@ def test_last_streaming_and_first_tiled_batch(ctx, T, flags):  # noqa: F811
                 tol=BF16_CLASS if flags else FP32_CLASS, flags=flags)
 
 
-@pytest.mark.parametrize("T,larger,flags", [(832, 1024, 0),
-                                            (608, 672, BF16)],
-                         ids=["fp32-class", "bf16-activations"])
-def test_wide_layer_takes_the_tiles(ctx, T, larger, flags):  # noqa: F811
-    """A wide layer (23 M multiply-adds a token; the streaming kernel was up to
-    70% slower on such layers) runs on the 256 x 256 tiles at T tokens, as it
+@pytest.mark.parametrize("H,T,larger,flags", [(2048, 832, 1024, 0), (2048, 608, 672, BF16),
+                                              (4096, 190, 1024, 0), (4096, 190, 1024, BF16)],
+                         ids=["fp32-class", "bf16-activations", "wider", "wider-bf16-activations"])
+def test_wide_layer_takes_the_tiles(ctx, H, T, larger, flags):  # noqa: F811
+    """A wide layer (23 or 46 M multiply-adds a token; the streaming kernel was up
+    to 70% slower on such layers) runs on the 256 x 256 tiles at T tokens, as it
     does at `larger`, where every layer does: rows of the two batches have the
     same bits, since a tile sums a row's products in one order whatever the
-    batch (and the router splits its sums alike at both sizes: 4 ways at 817 to
-    1024 tokens, 6 at 577 to 672). The streaming kernel sums in another."""
-    H, inter, E, K = 2048, 1408, 8, 6
+    batch. So does the router: up to hidden 2048 it splits its sums alike at both
+    sizes (4 ways at 817 to 1024 tokens, 6 at 577 to 672), beyond not at all. The
+    streaming kernel sums in another order."""
+    inter, E, K = 1408, 8, 6
     w = syn.moe_weights_device(H, inter, E, 2, seed=71)
     torch.cuda.synchronize()  # the library copies on its own stream
     layer = um.MoeLayer(ctx, um.config(H, inter, E, 2, K), w, um.MEMORY_DEVICE)
@@ -65,7 +66,7 @@ def test_wide_layer_takes_the_tiles(ctx, T, larger, flags):  # noqa: F811
     x = torch.randn((larger, H), generator=g, device="cuda")
     y, part = torch.empty_like(x), torch.empty((T, H), device="cuda")
     torch.cuda.synchronize()
-    print(f"wide layer T={T} against {larger} flags={flags}", flush=True)
+    print(f"wide layer H={H} T={T} against {larger} flags={flags}", flush=True)
     um.forward(ctx, layer, x, y, flags)
     um.forward(ctx, layer, x[:T].contiguous(), part, flags)
     layer.close()
